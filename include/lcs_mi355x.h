@@ -426,7 +426,7 @@ int lcs_batch_set_persistent(lcs_batch *batch, int cus);
  * depend on the tiling; the logged divergence and forcing power are sums of
  * per-tile partials, so their last bits do.  It then picks the fused RHS's
  * tile shape per class the same way (lcs_batch_set_rhs_tiles), timing
- * stage 1's RHS written into the spare arrays.  Synchronises; the next step
+ * stage 1's RHS written into the scratch arrays.  Synchronises; the next step
  * rebuilds the batch's tables and graphs. */
 int lcs_batch_autotune(lcs_batch *batch);
 /* Sets the tiling of the size class of box `index` (order of addition);
@@ -437,7 +437,7 @@ int lcs_batch_get_tiles(lcs_batch *batch, int index, int *tx, int *ty, int *zchu
 /* No counterpart in the reference.  The fused RHS tile of the size class of
  * box `index`: FP32 32x8 (default), 64x8, 64x16 or 32x16; FP64 32x4
  * (default), 32x8 or 64x8.  lcs_batch_autotune also picks it per class, by
- * timing stage 1's RHS into the boxes' spare arrays (no box changes).  Fields
+ * timing stage 1's RHS into the boxes' scratch arrays (no box changes).  Fields
  * do not depend on it. */
 int lcs_batch_set_rhs_tiles(lcs_batch *batch, int index, int tx, int ty);
 int lcs_batch_get_rhs_tiles(lcs_batch *batch, int index, int *tx, int *ty);

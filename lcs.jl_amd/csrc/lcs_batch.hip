@@ -194,12 +194,12 @@ static int rhs_shape(const Batch &B, const Geom &g)
 }
 
 // the fused RHS of a stage over every box, one launch per tile shape in use
-static int b_rhs(Batch &B, int stage, bool spare_out = false)
+static int b_rhs(Batch &B, int stage, bool scratch_out = false)
 {
     for (int q = 0; q < batch_rhs_shapes(B.esize); q++) {
         const int *sh = batch_rhs_shape(B.esize, q);
         int rc = launch_b_rhs(B.stream, B.esize, sh[0], sh[1], B.tab.d, B.rhs_tiles[q].d, B.rhs_tiles[q].n, stage,
-                              spare_out);
+                              scratch_out);
         if (rc) return rc;
     }
     return LCS_OK;
@@ -249,9 +249,7 @@ static void refresh_record(Batch &B, int i)
     Box &b = *B.boxes[i];
     BoxRec &r = B.tab_h[i];
     for (int q = 0; q < 7; q++) r.f[q] = b.f[q];
-    // a box in divergence form has no ping-pong partners; its D and F arrays
-    // serve where scratch of a field's size is written (RHS timing)
-    for (int q = 0; q < 4; q++) r.spare[q] = r.dv ? (char *)r.dv_mem + (size_t)q * r.dv_set * b.esize : b.spare[q];
+    for (int q = 0; q < 4; q++) r.spare[q] = b.spare[q];
     for (int q = 0; q < (int)b.profiles.size(); q++)
         for (int k = 0; k < LCS_N_PROPERTIES; k++) r.prof[q].props[k] = b.profiles[q].props[k];
 }
@@ -1030,7 +1028,7 @@ static int time_group_sweeps(Batch &B, int reps, hipEvent_t e0, hipEvent_t e1, f
 }
 
 // Fastest of `reps` runs of stage 1's fused RHS over the whole batch with the
-// current RHS tiling, written to the boxes' spare arrays: no box changes.
+// current RHS tiling, written to the boxes' scratch arrays: no box changes.
 static int time_rhs(Batch &B, int reps, hipEvent_t e0, hipEvent_t e1, float &best)
 {
     int rc;

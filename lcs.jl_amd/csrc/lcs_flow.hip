@@ -2541,7 +2541,9 @@ __global__ void __launch_bounds__(256) k_b_ghost_fill(const BoxRec *tab, const W
     const WorkItem w = work[blockIdx.x];
     const BoxRec &B = tab[w.box];
     if (b_halted(B)) return;
-    if (hsmac && B.S->hs_done) return;
+    // an HSMAC fill is for the boxes that sweep in place: in divergence form
+    // hs_par names a (D, F) set, and the ghosts are filled by the form itself
+    if (hsmac && (B.S->hs_done || B.dv)) return;
     const bool alt = hsmac && B.S->hs_par;
     const Geom g = B.g;
     long cz, cy, cx;
@@ -2705,9 +2707,16 @@ int launch_b_lf(hipStream_t s, int esize, const BoxRec *tab, const WorkItem *row
     return LCS_OK;
 }
 
+// an array of a field's size that holds nothing between HSMAC calls: D0, D1, F0
+// of a box in divergence form (which has no ping-pong partners), else a partner
+__device__ inline void *b_scratch(const BoxRec &B, int q, int esize)
+{
+    return B.dv ? (char *)B.dv_mem + (size_t)q * B.dv_set * esize : B.spare[q];
+}
+
 // fused RHS + update of one stage for every box
 template <typename T, int TX, int TY, bool BASE>
-__global__ void __launch_bounds__(TX *TY) k_b_rhs_flux(const BoxRec *tab, const TileItem *tiles, int spare_out)
+__global__ void __launch_bounds__(TX *TY) k_b_rhs_flux(const BoxRec *tab, const TileItem *tiles, int scratch_out)
 {
     extern __shared__ __align__(16) unsigned char rhs_lds_raw[];
     const TileItem t = tiles[blockIdx.x];
@@ -2721,7 +2730,7 @@ __global__ void __launch_bounds__(TX *TY) k_b_rhs_flux(const BoxRec *tab, const 
     a.W = (const T *)B.f[in + 2];
     a.P = (const T *)B.f[6];
     for (int q = 0; q < 3; q++) {
-        a.out[q] = spare_out ? (T *)B.spare[q] : (T *)B.f[(BASE ? 0 : 3) + q];
+        a.out[q] = scratch_out ? (T *)b_scratch(B, q, (int)sizeof(T)) : (T *)B.f[(BASE ? 0 : 3) + q];
         a.base[q] = BASE ? (const T *)B.f[q] : nullptr;
         a.di[q] = T(B.rhs_di[q]);
         a.di2[q] = T(B.rhs_di2[q]);
@@ -2733,7 +2742,7 @@ __global__ void __launch_bounds__(TX *TY) k_b_rhs_flux(const BoxRec *tab, const 
 }
 
 template <typename T, int TX, int TY>
-static int b_rhs_t(hipStream_t s, const BoxRec *tab, const TileItem *tiles, int ntiles, int stage, int spare_out)
+static int b_rhs_t(hipStream_t s, const BoxRec *tab, const TileItem *tiles, int ntiles, int stage, int scratch_out)
 {
     using Tile = RhsFlux<T, TX, TY, true>;
     const size_t lds = Tile::LDS_ELEMS * sizeof(T);
@@ -2741,16 +2750,16 @@ static int b_rhs_t(hipStream_t s, const BoxRec *tab, const TileItem *tiles, int 
     auto *k = stage == 2 ? k_b_rhs_flux<T, TX, TY, true> : k_b_rhs_flux<T, TX, TY, false>;
     int rc = kernel_setup((const void *)k, TX * TY, lds, nullptr);
     if (rc) return rc;
-    hipLaunchKernelGGL(k, dim3(ntiles), dim3(TX * TY), lds, s, tab, tiles, spare_out);
+    hipLaunchKernelGGL(k, dim3(ntiles), dim3(TX * TY), lds, s, tab, tiles, scratch_out);
     LCS_HIP(hipGetLastError());
     return LCS_OK;
 }
 
 int launch_b_rhs(hipStream_t s, int esize, int tx, int ty, const BoxRec *tab, const TileItem *tiles, int ntiles,
-                 int stage, bool spare_out)
+                 int stage, bool scratch_out)
 {
     if (ntiles == 0) return LCS_OK;
-    const int so = spare_out ? 1 : 0;
+    const int so = scratch_out ? 1 : 0;
     if (esize == 8) {
         if (tx == 32 && ty == 4) return b_rhs_t<double, 32, 4>(s, tab, tiles, ntiles, stage, so);
         if (tx == 32 && ty == 8) return b_rhs_t<double, 32, 8>(s, tab, tiles, ntiles, stage, so);

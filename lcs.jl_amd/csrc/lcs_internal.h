@@ -365,10 +365,10 @@ int launch_b_rcf(hipStream_t s, int esize, const BoxRec *tab, const WorkItem *me
 int rcf_prepare(Box &b, int kmin, int kmax, int c);
 int rcf_apply_blocks(const Box &b);
 int rcf_crop_slots(int kmax);
-// tiles of one shape (tx x ty, batch_rhs_shape); spare_out: write the result
-// to the boxes' spare arrays instead of the stage's output (for timing)
+// tiles of one shape (tx x ty, batch_rhs_shape); scratch_out: write the result
+// to the boxes' scratch arrays (b_scratch) instead of the stage's output (for timing)
 int launch_b_rhs(hipStream_t s, int esize, int tx, int ty, const BoxRec *tab, const TileItem *tiles, int ntiles,
-                 int stage, bool spare_out = false);
+                 int stage, bool scratch_out = false);
 // tx: tile width of the fused sweep (32 or 64); the tiles listed must all be of that width
 // force: boxes with lf_force apply the linear forcing of S->lf on load and
 // leave their per-tile power in part[kPowerSlot]

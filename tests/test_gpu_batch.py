@@ -250,3 +250,40 @@ def test_batch_tiling_changes_no_result(dtype):
         bt.set_rhs_tiles(0, 128, 8)
     bt.close()
     bd.close()
+
+
+def test_ghost_fill_of_a_thin_box_leaves_other_boxes_alone():
+    """A box thinner than the halo (8 cells, halo 9) makes the batch fill ghosts
+    before each in-place HSMAC group (its ghosts have several images).  That
+    fill must not touch a box in divergence form: here one whose D and F rows
+    are padded (sx >= 256), in four groups that each flip its parity (epsp 0: no
+    box ends early).  Its result is the one it has alone, bit for bit."""
+    import dataclasses
+
+    import lcs_mi355x as L
+    from lcs_mi355x import config as C
+    hs = C.HSMAC(True, True, "red-black-fast", 1.7, 0.0, 0, 12)
+
+    def cfg(dims):
+        c = c1_config(dims=dims, dtype="f32", profiles=0)
+        return dataclasses.replace(c, flow=dataclasses.replace(c.flow, couple=hs))
+
+    def build(c):
+        rng = np.random.default_rng(1)
+        box = L.Box(c.grid.dims, 9, c.flow.params, np.float32)
+        for name in ("U", "V", "W", "P"):
+            box.upload(name, rng.standard_normal(box.shape).astype(np.float32))
+        return box
+
+    wide, thin = cfg((240, 10, 12)), cfg((8, 16, 16))
+    alone, mixed, other = build(wide), build(wide), build(thin)
+    b1, b2 = L.Batch(), L.Batch()
+    b1.add(alone, L.step_config(wide))
+    b2.add(mixed, L.step_config(wide))
+    b2.add(other, L.step_config(thin))
+    for s in range(4):
+        assert b1.step()[0] == b2.step()[0], s
+        for name in ("U", "V", "W", "P"):
+            np.testing.assert_array_equal(mixed.download(name), alone.download(name), err_msg=f"step {s} {name}")
+    b1.close()
+    b2.close()
