@@ -291,7 +291,7 @@ static int rebuild(Batch &B)
     std::vector<TileItem> rtiles[kBatchRhsShapesMax], htiles[4];
     DvWork dvw;
     B.in_place = false;
-    auto in_div = [&](const Box &b) { return hsmac_takes_div(b.g, B.hs); };
+    auto in_div = [&](const Box &b) { return hsmac_takes_div(b.g, b.esize, B.hs); };
     const int domain = B.hs.time_blocking ? 1 : 3;
     B.xface = n > 0;
     for (int i = 0; i < n; i++) {
@@ -1071,7 +1071,7 @@ static int batch_autotune(Batch &B)
     for (int round = 0; round < 2 && rc == LCS_OK; round++)
         for (const auto &c : classes) {
             // (boxes in divergence form have tiles of their own)
-            if (hsmac_takes_div(make_geom(c[0], c[1], c[2], B.boxes[0]->g.h), B.hs)) continue;
+            if (hsmac_takes_div(make_geom(c[0], c[1], c[2], B.boxes[0]->g.h), B.esize, B.hs)) continue;
             std::array<int, 2> best = B.sweep_tune[c];
             float best_ms = 0;
             B.dirty = true;

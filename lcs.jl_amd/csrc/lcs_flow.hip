@@ -1264,7 +1264,7 @@ int launch_hsmac(Box &b, void **Us, DtRef dt, const lcs_hsmac_params &prm, int s
         return fail(LCS_ERR_INVALID, "unsupported coloring");
     if (prm.itrmax < 0 || prm.itrmin < 0) return fail(LCS_ERR_INVALID, "itrmin/itrmax must be >= 0");
     if (lf_deferred && prm.itrmax < 1) return fail(LCS_ERR_INVALID, "deferred forcing needs a sweep");
-    if (hsmac_takes_div(b.g, prm)) return launch_hsmac_div(b, Us, dt, prm, slot, lf_deferred);
+    if (hsmac_takes_div(b.g, b.esize, prm)) return launch_hsmac_div(b, Us, dt, prm, slot, lf_deferred);
     return b.esize == 8 ? hsmac_t<double>(b, Us, dt, prm, slot, lf_deferred)
                         : hsmac_t<float>(b, Us, dt, prm, slot, lf_deferred);
 }

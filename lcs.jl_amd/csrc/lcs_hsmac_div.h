@@ -35,6 +35,7 @@
 #pragma once
 
 #include "lcs_device.h"
+#include "lcs_hsmac_plan.h"
 #include "lcs_hsmac_tile.h"
 #include "lcs_internal.h"
 
@@ -91,55 +92,6 @@ template <typename T>
 __device__ inline T dv_self(const DvCoef<T> &c, T d, T dp)
 {
     return __builtin_elementwise_fma(c.c0, dp, __builtin_elementwise_fma(c.c0l, dp, d));
-}
-
-// Row pitch of D and F in elements: rows start on 64-byte lines, and the pitch
-// is an odd number of lines, so that the rows of a tile spread over the memory
-// channels (a pitch of 4096 bytes ran a marching copy at 3.4 TB/s, 4032 bytes
-// at 4.7, the field's own 4024 at 3.5: 1006^3 FP32, 112-wide tiles).
-__host__ __device__ inline int dv_pitch(const Geom &g, int esize)
-{
-    if (g.sx < 256) return (int)g.sx;  // small boxes run from cache
-    const int line = 64 / esize, n = ((int)g.sx + line - 1) / line;
-    return (n | 1) * line;
-}
-
-// seam and edge planes of a box, one allocation: U, V, W seam planes over
-// the interior, then U, V, W edge planes over the whole cross-section
-struct DvPlanes {
-    long seam[3], edge[3], dp[3];
-    long total;
-};
-__host__ __device__ inline DvPlanes dv_planes(const Geom &g)
-{
-    DvPlanes p;
-    const long nx = g.nx, ny = g.ny, nz = g.nz, sz = nz + 2 * g.h;
-    long at = 0;
-    const long s[3] = {ny * nz, nx * nz, nx * ny}, e[3] = {g.sy * sz, g.sx * sz, g.sx * g.sy};
-    // corrections of the face slabs of the overlap order, x, y, z: 2 slabs x 3 layers
-    const long d[3] = {6 * (ny - 1) * (nz - 1), 6 * (nx + 5) * (nz - 1), 6 * (nx + 5) * (ny + 5)};
-    for (int a = 0; a < 3; a++) {
-        p.seam[a] = at;
-        at += s[a];
-    }
-    for (int a = 0; a < 3; a++) {
-        p.edge[a] = at;
-        at += e[a];
-    }
-    for (int a = 0; a < 3; a++) {
-        p.dp[a] = at;
-        at += d[a];
-    }
-    p.total = at;
-    return p;
-}
-
-// boxes the divergence form takes: one image per ghost, and face slabs of
-// one axis (with the ring of cells they change) that do not meet
-__host__ __device__ inline bool dv_fits(const Geom &g)
-{
-    const int m = g.h > 8 ? g.h : 8;
-    return g.h >= 3 && g.nx >= m && g.ny >= m && g.nz >= m;
 }
 
 enum { kDvPlain = 0, kDvConstruct = 1 };
@@ -251,24 +203,16 @@ __device__ inline DvPair<T> dv_load2(const T *p)
 // 64-byte line, so stored row segments start and end on lines.
 template <typename T, int NS, int MODE, int LX, int RW, int NB, int PF = 2>
 struct DvTile {
-    static constexpr int LINE = 64 / (int)sizeof(T);
-    static constexpr int W = 2 * LX, OWN = (W - 4 * NS) / LINE * LINE, HX = (W - OWN) / 2;
-    static constexpr int ROWS = NB * RW, HY = 2 * NS, HZ = 2 * NS, NT = NB * LX;
+    using Win = DvWindow<(int)sizeof(T), NS, LX, RW, NB>;
+    static constexpr int W = Win::W, OWN = Win::OWN, HX = Win::HX;
+    static constexpr int ROWS = Win::ROWS, HY = Win::HY, HZ = 2 * NS, NT = NB * LX;
     static constexpr int EX = 2 * NS * 2 * NB * 2 * LX;  // exchange elements in LDS
     static_assert(RW % 2 == 0, "a block's first row keeps the parity of the tile's");
     static_assert(PF % 2 == 0, "a register set serves steps of one parity");
     static_assert(HX >= 2 * NS && HX % 2 == 0, "halo of the window");
 
-    // one element of padding at the end keeps the last window's edge outside the array
-    __host__ __device__ static int tiles_x(const Geom &g)
-    {
-        return g.sx + 1 <= W ? 1 : ((int)g.sx + OWN - 1) / OWN;
-    }
-    __host__ __device__ static int tiles_y(const Geom &g)
-    {
-        const int s = (int)g.sy + 1, own = ROWS - 2 * HY;
-        return s <= ROWS ? 1 : 1 + (s - ROWS + own - 1) / own;
-    }
+    __host__ __device__ static int tiles_x(const Geom &g) { return Win::tiles_x(g); }
+    __host__ __device__ static int tiles_y(const Geom &g) { return Win::tiles_y(g); }
 
     struct Th {
         int X, xo, b, lx;       // first cell of the lane, clamped load offset, block, lane

@@ -46,16 +46,7 @@ __global__ void __launch_bounds__(LX *NB)
 }
 
 // ---- refresh --------------------------------------------------------------------
-// one thread per cell of the shell: z planes 0..h and nz+h-1.., then rows y
-// 0..h and ny+h-1.., then x 0..h and nx+h-1..  (2h+2 layers on each axis)
-__host__ __device__ inline void dv_refresh_cells(const Geom &g, long n[3])
-{
-    const long L = 2 * g.h + 2;
-    n[0] = L * g.sx * g.sy;
-    n[1] = L * g.sx * (g.nz - 2);
-    n[2] = L * (g.ny - 2) * (long)(g.nz - 2);
-}
-
+// one thread per cell of the shell (dv_refresh_cells)
 template <typename T>
 __device__ inline void dv_refresh_block(const Geom &g, const DvCoef<T> &c, const T *Do, const T *Fo, T *Dn, T *Fn, T *P,
                                         T *planes, T dti, int accumulate, int blk)
@@ -147,16 +138,16 @@ struct DvFaces {
 };
 
 template <typename T, int AXIS>
-__device__ inline double dv_face_block(const DvFaces<T> &f, const T *D, const DvCoef<T> &c, int want_sum, int blk)
+__device__ inline double dv_face_block(const DvFaces<T> &f, const T *D, const DvCoef<T> &c, int want_sum, int blk,
+                                       int nblk)
 {
     const Geom &g = f.g;
     // lateral ranges: l1 is the unit-stride index of the buffer
     const int lo1 = AXIS == 2 ? 2 : -1, hi1 = AXIS == 2 ? g.ny : g.nx + 3;
     const int lo2 = AXIS == 0 ? -1 : 2, hi2 = AXIS == 0 ? g.ny + 3 : g.nz;
     const int n1 = hi1 - lo1 + 1, n2 = hi2 - lo2 + 1, n = AXIS == 0 ? g.nz : (AXIS == 1 ? g.ny : g.nx);
-    const int t0 = blk * 256 + (int)threadIdx.x;
     double acc = 0.0;
-    if (t0 < 2 * n1 * n2) {
+    for (int t0 = blk * 256 + (int)threadIdx.x; t0 < 2 * n1 * n2; t0 += nblk * 256) {
         const int s = t0 >= n1 * n2, u = s ? t0 - n1 * n2 : t0;
         const int l1 = lo1 + u % n1, l2 = lo2 + u / n1;
         const T ca = AXIS == 0 ? c.cz : (AXIS == 1 ? c.cy : c.cx);
@@ -255,22 +246,14 @@ __global__ void __launch_bounds__(256)
 {
     __shared__ double lds[16];
     if (S->hs_done) return;
-    const double acc = dv_face_block<T, AXIS>(f, D, c, want_sum, (int)blockIdx.x);
+    const double acc = dv_face_block<T, AXIS>(f, D, c, want_sum, (int)blockIdx.x, (int)gridDim.x);
     if (want_sum) {
         const double v = block_sum(acc, lds);
         if (threadIdx.x == 0) part[blockIdx.x] = v;
     }
 }
 
-// cells a slab correction changes, each handled once: layers -1..2 and n..n+3
-// of z over domain 1, then of y for k in 3..nz-1, then of x for j, k inside
-__host__ __device__ inline void dv_face_cells(const Geom &g, long n[3])
-{
-    n[0] = 8L * (g.nx + 5) * (g.ny + 5);
-    n[1] = 8L * (g.nx + 5) * (g.nz - 3);
-    n[2] = 8L * (g.ny - 3) * (g.nz - 3);
-}
-
+// one thread per cell that a slab correction changes (dv_face_cells)
 template <typename T>
 __device__ inline void dv_apply_block(const DvFaces<T> &f, T *D, T *F, const DvCoef<T> &c, int blk)
 {
@@ -349,12 +332,13 @@ __global__ void k_dv_check(const double *part, DvCheck a, DevScalars *S)
 // U += dxi (F(i) - F(i+1)) and likewise V, W; P += F / dt; over the whole
 // array, with the seam and edge planes.  FORCE applies the deferred linear
 // forcing to the velocity first and sums its power over the interior.  Each
-// thread marches a column of planes, F of the plane above in a register.
+// thread marches a column of planes, F of the plane above in a register; a
+// workgroup takes the tasks (column, chunk) t, t + nblk, ...
 // when: 0 always, 1 only if the call has converged
 template <typename T, bool FORCE>
-__device__ inline double dv_finish_block(const Geom &g, T *U, T *V, T *W, T *P, const T *F, const T *planes,
-                                         const DvCoef<T> &c, double d, const DevScalars *S, int seams, int zc, int gxy,
-                                         int t)
+__device__ inline double dv_finish_task(const Geom &g, T *U, T *V, T *W, T *P, const T *F, const T *planes,
+                                        const DvCoef<T> &c, double d, const DevScalars *S, int seams, int zc, int gxy,
+                                        int t)
 {
     const T dti = T(1.0 / d);
     const DvPlanes pl = dv_planes(g);
@@ -414,6 +398,18 @@ __device__ inline double dv_finish_block(const Geom &g, T *U, T *V, T *W, T *P, 
 }
 
 template <typename T, bool FORCE>
+__device__ inline double dv_finish_block(const Geom &g, T *U, T *V, T *W, T *P, const T *F, const T *planes,
+                                         const DvCoef<T> &c, double d, const DevScalars *S, int seams, int zc, int gxy,
+                                         int blk, int nblk)
+{
+    const int ntask = gxy * ((g.nz + 2 * g.h + zc - 1) / zc);
+    double pw = 0.0;
+    for (int t = blk; t < ntask; t += nblk)
+        pw += dv_finish_task<T, FORCE>(g, U, V, W, P, F, planes, c, d, S, seams, zc, gxy, t);
+    return pw;
+}
+
+template <typename T, bool FORCE>
 __global__ void __launch_bounds__(256)
     k_dv_finish(Geom g, T *U, T *V, T *W, T *P, DvSets<T> sets, const T *planes, DvCoef<T> c, DtRef dt,
                 DevScalars *S, int when, int par, int slot, int seams, int zc, int gxy, double *part)
@@ -423,7 +419,7 @@ __global__ void __launch_bounds__(256)
     if (when == 1 && !done) return;
     const double pw = dv_finish_block<T, FORCE>(g, U, V, W, P, sets.F[done ? S->hs_par : par], planes, c,
                                                 dt.factor * (*dt.src), S, seams, zc, gxy,
-                                                xcd_linear(blockIdx.x, gridDim.x));
+                                                xcd_linear(blockIdx.x, gridDim.x), (int)gridDim.x);
     if (FORCE) {
         const double v = block_sum(pw, lds);
         if (threadIdx.x == 0) part[blockIdx.x] = v;
@@ -444,19 +440,6 @@ __global__ void k_dv_power(const double *part, int nblk, double len, DevScalars 
     if (threadIdx.x == 0) S->p = s / len;
 }
 
-// columns of planes: short ones where the grid is small, so that the chip is
-// filled, and at most 32 planes
-static void dv_finish_grid(const Geom &g, int cus, int &gxy, int &zc, int &blocks)
-{
-    const int nplanes = g.nz + 2 * g.h;
-    gxy = (int)((g.sx * g.sy + 255) / 256);
-    int nz = (int)std::min<long>(nplanes, std::max<long>(1, (8L * cus + gxy - 1) / gxy));
-    nz = std::max(nz, (nplanes + 31) / 32);
-    nz = std::min<int>(nz, std::max(1, kMaxPartBlocks / gxy));
-    zc = (nplanes + nz - 1) / nz;
-    blocks = gxy * ((nplanes + zc - 1) / zc);
-}
-
 // ---- one call ------------------------------------------------------------------
 template <typename T>
 struct DvRun {
@@ -470,27 +453,6 @@ struct DvRun {
     int nrefresh = 0;  // refreshes so far
     bool force = false;
     DvCheck ck;
-
-    // z-chunks of a sweep: the count with the fewest plane-steps on the
-    // busiest CU, a chunk paying 4 NS halo planes, among chunks of at most
-    // kMaxChunk planes: workgroups end at different times, and short chunks
-    // even that out (1000^3, two sweeps: 4.17 ms with 2 chunks, 3.92 with 8)
-    static constexpr int kMaxChunk = 128;
-    static int chunks(long cols, int nplanes, int halo, long slots, int cap)
-    {
-        const int n0 = (nplanes + kMaxChunk - 1) / kMaxChunk;
-        int best_n = std::max(1, (int)std::min<long>(n0, cap / cols));
-        double best = 1e300;
-        for (int n = best_n; n <= nplanes && cols * n <= cap; n++) {
-            const int zc = (nplanes + n - 1) / n;
-            const double cost = (double)((cols * n + slots - 1) / slots) * (zc + halo + 2);
-            if (cost < best * 0.999) {
-                best = cost;
-                best_n = n;
-            }
-        }
-        return best_n;
-    }
 
     template <int NS, int MODE, int LX, int RW, int NB, int PF = 2>
     int sweep(int k0, int k1, int sum0, int sum1)
@@ -507,7 +469,7 @@ struct DvRun {
         a.U = U;
         a.V = V;
         a.W = W;
-            a.c = c;
+        a.c = c;
         a.px = dv_pitch(g, (int)sizeof(T));
         a.kind[0] = k0;
         a.kind[1] = k1;
@@ -515,11 +477,10 @@ struct DvRun {
         a.sum[1] = sum1;
         const int gx = Tile::tiles_x(g), gy = Tile::tiles_y(g), nplanes = g.nz + 2 * g.h;
         const long cols = (long)gx * gy;
-        if (cols > kMaxPartBlocks) return fail(LCS_ERR_INVALID, "grid too large for the HSMAC sweep");
         const void *k = (const void *)k_dv_sweep<T, NS, MODE, LX, RW, NB, PF>;
         int per_cu = 1, rc = kernel_setup(k, Tile::NT, 0, &per_cu);
         if (rc) return rc;
-        int nz = chunks(cols, nplanes, 4 * NS, (long)b.cus * per_cu, kMaxPartBlocks);
+        int nz = dv_chunks(cols, nplanes, 4 * NS, (long)b.cus * per_cu);
         a.zc = (nplanes + nz - 1) / nz;
         nz = (nplanes + a.zc - 1) / a.zc;
         const int blocks = (int)(cols * nz);
@@ -576,11 +537,11 @@ struct DvRun {
         const Geom &g = b.g;
         DvFaces<T> f{g, planes, dv_planes(g), dv_pitch(g, (int)sizeof(T))};
         T *D = sets.D[par], *F = sets.F[par];
-        const long cols[3] = {2L * (g.nx + 5) * (g.ny + 5), 2L * (g.nx + 5) * (g.nz - 1), 2L * (g.ny - 1) * (g.nz - 1)};
+        long cols[3];
+        dv_face_columns(g, cols);
         ProfScope ps(b, "hsmac_faces", 0.0);
         for (int ax = 0; ax < 3; ax++) {
-            const int blocks = (int)((cols[ax] + 255) / 256);
-            if (blocks > kMaxPartBlocks) return fail(LCS_ERR_INVALID, "grid too large for the HSMAC face slabs");
+            const int blocks = dv_blocks(cols[ax]);
             double *part = b.part + (long)ck.npass * kMaxPartBlocks;
             if (ax == 0)
                 hipLaunchKernelGGL((k_dv_face<T, 0>), dim3(blocks), dim3(256), 0, b.stream, f, D, c, b.S, want_sum, part);
@@ -613,7 +574,6 @@ struct DvRun {
         const Geom &g = b.g;
         int gxy, zc, blocks;
         dv_finish_grid(g, b.cus, gxy, zc, blocks);
-        if (blocks > kMaxPartBlocks) return fail(LCS_ERR_INVALID, "grid too large for the HSMAC update");
         double *part = b.part + kPowerSlot;
         {
             ProfScope ps(b, "hsmac_finish", 9.0 * sizeof(T) * g.cells());
@@ -640,17 +600,11 @@ struct DvRun {
     }
 };
 
-// elements of one D or F array, a multiple of a line
-static size_t dv_elems(const Geom &g, size_t esize)
-{
-    return (size_t)dv_pitch(g, (int)esize) * (size_t)g.sy * (size_t)(g.nz + 2 * g.h);
-}
-
 // the box's D and F sets and planes: one allocation, made by the first call
 int dv_buffers(Box &b)
 {
     if (b.dv) return LCS_OK;
-    const size_t bytes = (4 * dv_elems(b.g, b.esize) + (size_t)dv_planes(b.g).total) * b.esize;
+    const size_t bytes = dv_bytes(b.g, b.esize);
     LCS_HIP(hipMalloc(&b.dv, bytes));
     b.bytes += bytes;
     return LCS_OK;
@@ -739,11 +693,11 @@ int launch_hsmac_div(Box &b, void **Us, DtRef dt, const lcs_hsmac_params &prm, i
                         : hsmac_div_t<float>(b, Us, dt, prm, slot, lf_deferred);
 }
 
-bool hsmac_takes_div(const Geom &g, const lcs_hsmac_params &prm)
+bool hsmac_takes_div(const Geom &g, int esize, const lcs_hsmac_params &prm)
 {
-    return prm.time_blocking && prm.overlap && prm.coloring == LCS_COLORING_RED_BLACK_FAST && prm.itrmax >= 1 && dv_fits(g);
+    return prm.time_blocking && prm.overlap && prm.coloring == LCS_COLORING_RED_BLACK_FAST && prm.itrmax >= 1 &&
+           dv_fits(g, esize);
 }
-
 
 // ---- batches -------------------------------------------------------------------
 // The same per box, one launch per phase over the listed boxes.  A box's two
@@ -831,7 +785,8 @@ __global__ void __launch_bounds__(256) k_b_dv_face(const BoxRec *tab, const Work
     const WorkItem w = work[blockIdx.x];
     const BoxRec &B = tab[w.box];
     if (b_halted(B) || B.S->hs_done) return;
-    const double acc = dv_face_block<T, AXIS>(dv_b_faces<T>(B), dv_b_set<T>(B, 0, cur), dv_coef_rec<T>(B), sum, w.blk);
+    const double acc = dv_face_block<T, AXIS>(dv_b_faces<T>(B), dv_b_set<T>(B, 0, cur), dv_coef_rec<T>(B), sum, w.blk,
+                                              B.dv_faces[AXIS]);
     if (sum) {
         const double v = block_sum(acc, lds);
         if (threadIdx.x == 0) B.part[(long)(2 + AXIS) * kMaxPartBlocks + w.blk] = v;
@@ -906,11 +861,12 @@ __global__ void __launch_bounds__(256)
     const double d = dtfac * B.S->dt;
     if (forced) {
         const double pw =
-            dv_finish_block<T, true>(B.g, U, V, W, P, F, planes, c, d, B.S, seams, B.dv_fzc, B.dv_gxy, w.blk);
+            dv_finish_block<T, true>(B.g, U, V, W, P, F, planes, c, d, B.S, seams, B.dv_fzc, B.dv_gxy, w.blk,
+                                     B.dv_fin);
         const double v = block_sum(pw, lds);
         if (threadIdx.x == 0) B.part[kPowerSlot + w.blk] = v;
     } else
-        dv_finish_block<T, false>(B.g, U, V, W, P, F, planes, c, d, B.S, seams, B.dv_fzc, B.dv_gxy, w.blk);
+        dv_finish_block<T, false>(B.g, U, V, W, P, F, planes, c, d, B.S, seams, B.dv_fzc, B.dv_gxy, w.blk, B.dv_fin);
 }
 
 __global__ void k_b_dv_power(const BoxRec *tab, const int *boxes, int final, int ngroups, int force)
@@ -923,15 +879,6 @@ __global__ void k_b_dv_power(const BoxRec *tab, const int *boxes, int final, int
     for (int q = threadIdx.x; q < B.dv_fin; q += blockDim.x) v += B.part[kPowerSlot + q];
     v = block_sum(v, lds);
     if (threadIdx.x == 0) B.S->p = v / (double)B.g.cells();
-}
-
-// planes per chunk of a batched sweep: about eight chunks for small boxes, of
-// about 28 planes for others (each re-reads 4 NS planes; the launch fills the
-// chip with the tiles of many boxes)
-static int dv_batch_zc(int nplanes)
-{
-    const int n = nplanes <= 80 ? 8 : std::max(1, (nplanes + 14) / 28);
-    return (nplanes + n - 1) / n;
 }
 
 template <typename T>
@@ -970,9 +917,10 @@ static int dv_record_t(Box &b, const lcs_hsmac_params &prm, int i, BoxRec &r, Dv
     list(w.refresh, blocks(n[0] + n[1] + n[2]));
     dv_face_cells(g, n);
     list(w.apply, blocks(n[0] + n[1] + n[2]));
-    const long cols[3] = {2L * (g.nx + 5) * (g.ny + 5), 2L * (g.nx + 5) * (g.nz - 1), 2L * (g.ny - 1) * (g.nz - 1)};
+    long cols[3];
+    dv_face_columns(g, cols);
     for (int a = 0; a < 3; a++) {
-        r.dv_faces[a] = blocks(cols[a]);
+        r.dv_faces[a] = dv_blocks(cols[a]);
         list(w.faces[a], r.dv_faces[a]);
     }
     dv_finish_grid(g, 8, r.dv_gxy, r.dv_fzc, r.dv_fin);
@@ -980,9 +928,8 @@ static int dv_record_t(Box &b, const lcs_hsmac_params &prm, int i, BoxRec &r, Dv
     const long X = g.nx + 2L * g.h, Y = g.ny + 2L * g.h;
     list(w.ghost, blocks(2L * g.h * (X * Y + X * g.nz + (long)g.ny * g.nz)));
     w.boxes.push_back(i);
-    int most = std::max(std::max(r.dv_tiles[0], r.dv_tiles[1]), r.dv_fin);
-    for (int a = 0; a < 3; a++) most = std::max(most, r.dv_faces[a]);
-    return most > kMaxPartBlocks ? fail(LCS_ERR_CAPACITY, "box too large for a batch") : LCS_OK;
+    return std::max(r.dv_tiles[0], r.dv_tiles[1]) > kMaxPartBlocks ? fail(LCS_ERR_CAPACITY, "box too large for a batch")
+                                                                   : LCS_OK;
 }
 
 int dv_batch_record(Box &b, const lcs_hsmac_params &prm, int i, BoxRec &r, DvWork &w)

@@ -217,12 +217,12 @@ int launch_cfl(Box &b, double cfl, double dtmax, bool fill = true);  // writes S
 int launch_hsmac(Box &b, void **Us, DtRef dt, const lcs_hsmac_params &prm, int log_slot, bool lf_deferred = false);
 // the same in divergence form (lcs_hsmac_div.hip), for the calls it takes: time
 // blocking with overlap and red-black-fast, on boxes of at least 8 cells an
-// axis.  Acts in place; launch_hsmac hands such calls over.
+// axis (dv_fits, lcs_hsmac_plan.h).  Acts in place; launch_hsmac hands such calls over.
 int launch_hsmac_div(Box &b, void **Us, DtRef dt, const lcs_hsmac_params &prm, int log_slot, bool lf_deferred);
 int dv_buffers(Box &b);
 // groups after which a call carries its corrections into the velocity (dv_fits boxes)
 constexpr int kDvGroups = 8;
-bool hsmac_takes_div(const Geom &g, const lcs_hsmac_params &prm);
+bool hsmac_takes_div(const Geom &g, int esize, const lcs_hsmac_params &prm);
 int kernel_setup(const void *func, int threads, size_t lds, int *per_cu);
 int launch_force_linear(Box &b, double power, DtRef dt);  // writes S->lf, S->p
 // writes S->lf only; face_only: the means read the x = 0, y = 0, z = 0
