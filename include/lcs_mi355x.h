@@ -186,7 +186,11 @@ int lcs_update(lcs_box *box, int stage, double dt_stage);
 int lcs_rhs_update(lcs_box *box, int stage, double dt_stage);
 
 /* Flows.couple!(::HSMAC) (src/flows/couples/couple.jl:13-17,
- * src/flows/couples/hsmac.jl:52-201): stage 1 acts on Us2, stage 2 on Us */
+ * src/flows/couples/hsmac.jl:52-201): stage 1 acts on Us2, stage 2 on Us.
+ * With time blocking, overlap and red-black-fast the sweeps carry the divergence
+ * itself; *div and the test against epsp are then of that divergence and of the
+ * mean rounding error of the velocity in its type, added as squares, so that
+ * neither falls below what the returned velocity shows. */
 int lcs_hsmac(lcs_box *box, int stage, double dt_stage, const lcs_hsmac_params *params, int *itr,
               double *div);
 

@@ -32,6 +32,14 @@
 // (D, F) set to the other, and the refresh then corrects ghosts and low planes
 // of the sweep's output from the sweep's input: no thread reads what another
 // one writes.
+// The divergence a check sees is that of D, which the sweeps reduce far below
+// what the velocity can show: U rounded to its type has an error of ulp / sqrt(12)
+// a face, and ulp^2 averages 3/7 eps^2 U^2 over the mantissas, so a cell's
+// div^2 has the mean eps^2 / 14 (dxi^2 U^2 + dyi^2 V^2 + dzi^2 W^2) even where
+// D is zero.  The construct pass sums that term and every check adds it
+// (dv_noise): a call whose epsp lies below it runs to itrmax, as the sweeps on
+// the velocity do, and the logged divergence is one the velocity shows (64^3
+// FP32, U in [0, 1): floor 3.2e-8 / dx, the returned velocity's 2.5e-8 to 3e-8).
 #pragma once
 
 #include "lcs_device.h"
@@ -70,6 +78,13 @@ inline DvCoef<T> dv_coef(const Geom &g, double omega)
     c.c0l = T(s - (long double)c.c0);
     c.k = -T(omega) * (T(1) / c.c0);
     return c;
+}
+// the factor of the construct pass's sum in div^2 (see above)
+template <typename T>
+inline double dv_noise(const Geom &g)
+{
+    const double eps = sizeof(T) == 8 ? 0x1p-52 : 0x1p-23;
+    return eps * eps / 14.0 / (double)g.len;
 }
 // a batch record's coefficients (the T values, stored as doubles)
 template <typename T>
@@ -234,6 +249,7 @@ struct DvTile {
         T rp[NS][RW], rpp[NS][RW], bp[NS][RW], bpp[NS][RW];  // dp of the last planes
         T bout[RW], fr[RW];     // black D of the next output plane, red F of the next F plane
         double acc[NS];
+        T nse;  // construct: sum of dxi^2 U^2 + dyi^2 V^2 + dzi^2 W^2 (a lane that owns one of its rows counts both)
     };
 
     __device__ static inline int clampi(int v, int hi) { return v < 0 ? 0 : (v > hi ? hi : v); }
@@ -291,6 +307,7 @@ struct DvTile {
             if constexpr (MODE == kDvConstruct) th.wp[r].v[0] = th.wp[r].v[1] = z;
         }
         for (int q = 0; q < NS; q++) th.acc[q] = 0.0;
+        th.nse = T(0);
         return !(th.wx0 >= h + 1 && th.wx0 + W - 1 <= g.nx + h - 1 && th.wy0 >= h + 1 &&
                  th.wy0 + ROWS - 1 <= g.ny + h - 1);
     }
@@ -378,6 +395,7 @@ struct DvTile {
         T R[RW];
         // the loaded plane, red and black apart
         T bload[RW];
+        T nse = T(0);
 #pragma unroll
         for (int r = 0; r < RW; r++) {
             DvPair<T> d = th.d[SET][r];
@@ -390,11 +408,16 @@ struct DvTile {
                 d.v[1] = ((c.dxi * (u1 - u0) + c.dyi * (v1.v[1] - v0.v[1])) + c.dzi * (w1.v[1] - th.wp[r].v[1])) *
                          a.dscale;
                 th.wp[r] = w1;
+                const T e = (c.cx * (u0 * u0 + u1 * u1) + c.cy * (v1.v[0] * v1.v[0] + v1.v[1] * v1.v[1])) +
+                            c.cz * (w1.v[0] * w1.v[0] + w1.v[1] * w1.v[1]);
+                nse += e;
             }
             const int sr = (E + r) & 1;
             R[r] = d.v[sr];
             bload[r] = d.v[1 - sr];
         }
+        if constexpr (MODE == kDvConstruct)
+            if (q >= th.zo0 && q < th.zo1) th.nse += nse;
         load_d<EXY>(a, th, q + PF, SET);
         // plane of F handled at this step
         const int zf = q - 2 * (NS - 1) - 1;
@@ -566,8 +589,8 @@ struct DvTile {
         }
     }
 
-    // the tile's sweeps; sums of div^2 of the lane's cells in acc
-    __device__ static inline void run(const DvArgs<T> &a, int bx, int by, int bz, T *lds, double acc[NS])
+    // the tile's sweeps; sums of div^2 of the lane's cells in acc, and of the rounding term in nse
+    __device__ static inline void run(const DvArgs<T> &a, int bx, int by, int bz, T *lds, double acc[NS], double &nse)
     {
         Th th;
         const bool edge = init(a, bx, by, bz, th);
@@ -579,6 +602,7 @@ struct DvTile {
             march<false>(a, lds, th);
 #pragma unroll
         for (int s = 0; s < NS; s++) acc[s] = th.acc[s];
+        nse = th.own ? (double)th.nse : 0.0;
     }
 };
 

@@ -8,6 +8,11 @@
 
 namespace lcs {
 
+// Partial slots of a call: 0 and 1 the sums of div^2 of a pass's sweeps, 2 to 4
+// those of the face slabs, 5 the rounding terms of the construct pass, which
+// every check until the next one reads.
+constexpr long kDvNoiseSlot = 5L * kMaxPartBlocks;
+
 // ---- sweeps -------------------------------------------------------------------
 // the two (D, F) sets; which one is current is known on the host until the
 // call has converged
@@ -16,9 +21,11 @@ struct DvSets {
     T *D[2], *F[2];
 };
 
+// (The FP32 construct pass of 512 threads needs 129 registers left alone; at
+// 128 two workgroups share a CU, as before it summed the rounding terms.)
 template <typename T, int NS, int MODE, int LX, int RW, int NB, int PF>
-__global__ void __launch_bounds__(LX *NB)
-    k_dv_sweep(DvArgs<T> a, int gx, int gy, int force, DtRef dt, DevScalars *S, double *part0, double *part1)
+__global__ void __launch_bounds__(LX *NB, MODE == kDvConstruct && sizeof(T) == 4 ? 4 : 1)
+    k_dv_sweep(DvArgs<T> a, int gx, int gy, int force, DtRef dt, DevScalars *S, double *part)
 {
     using Tile = DvTile<T, NS, MODE, LX, RW, NB, PF>;
     __shared__ __align__(16) T lds[Tile::EX];
@@ -36,13 +43,17 @@ __global__ void __launch_bounds__(LX *NB)
         }
     }
     const int t = xcd_linear(blockIdx.x, gridDim.x);
-    double acc[NS];
-    Tile::run(a, t % gx, t / gx % gy, t / (gx * gy), lds, acc);
+    double acc[NS], nse;
+    Tile::run(a, t % gx, t / gx % gy, t / (gx * gy), lds, acc, nse);
     for (int s = 0; s < NS; s++)
         if (a.sum[s]) {
             const double v = block_sum(acc[s], red_lds);
-            if (threadIdx.x == 0) (s == 0 ? part0 : part1)[blockIdx.x] = v;
+            if (threadIdx.x == 0) part[(long)s * kMaxPartBlocks + blockIdx.x] = v;
         }
+    if (MODE == kDvConstruct) {
+        const double v = block_sum(nse, red_lds);
+        if (threadIdx.x == 0) part[kDvNoiseSlot + blockIdx.x] = v;
+    }
 }
 
 // ---- refresh --------------------------------------------------------------------
@@ -304,7 +315,9 @@ __global__ void __launch_bounds__(256) k_dv_face_apply(DvFaces<T> f, T *D, T *F,
 // ---- convergence ----------------------------------------------------------------
 struct DvCheck {
     int npass;
-    int cnt[6];
+    int cnt[5];
+    int nnoise;            // workgroups of the construct pass
+    double noise;          // dv_noise
     double len3, dxmin, epsp;
     int itr;     // index of the sweep
     int par;     // set that holds its result
@@ -314,13 +327,15 @@ struct DvCheck {
 __global__ void k_dv_check(const double *part, DvCheck a, DevScalars *S)
 {
     __shared__ double lds[16];
+    // (the first rounding term is loaded ahead of the flag's wait)
+    double acc = 0.0, nse = (int)threadIdx.x < a.nnoise ? part[kDvNoiseSlot + threadIdx.x] : 0.0;
     if (S->hs_done) return;
-    double acc = 0.0;
     for (int q = 0; q < a.npass; q++)
         for (int m = threadIdx.x; m < a.cnt[q]; m += blockDim.x) acc += part[(long)q * kMaxPartBlocks + m];
-    const double s = block_sum(acc, lds);
+    for (int m = threadIdx.x + blockDim.x; m < a.nnoise; m += blockDim.x) nse += part[kDvNoiseSlot + m];
+    const double s = block_sum(acc / a.len3 + a.noise * nse, lds);
     if (threadIdx.x == 0) {
-        const double div = sqrt(s / a.len3);
+        const double div = sqrt(s);
         S->hs_div = div;
         if (a.decide && div * a.dxmin < a.epsp) {
             S->hs_itr = a.itr;
@@ -491,8 +506,9 @@ struct DvRun {
         ProfScope ps(b, MODE == kDvConstruct ? "hsmac_construct" : (NS == 2 ? "hsmac_sweep2" : "hsmac_sweep"),
                      (MODE == kDvConstruct ? 5.0 : 4.0) * cells);
         hipLaunchKernelGGL((k_dv_sweep<T, NS, MODE, LX, RW, NB, PF>), dim3(blocks), dim3(Tile::NT), 0, b.stream, a, gx,
-                           gy, force ? 1 : 0, dt, b.S, b.part, b.part + kMaxPartBlocks);
+                           gy, force ? 1 : 0, dt, b.S, b.part);
         LCS_HIP(hipGetLastError());
+        if (MODE == kDvConstruct) ck.nnoise = blocks;
         ck.npass = 0;
         ck.cnt[ck.npass++] = sum0 ? blocks : 0;
         ck.cnt[ck.npass++] = sum1 ? blocks : 0;
@@ -640,6 +656,7 @@ static int hsmac_div_t(Box &b, void **Us, DtRef dt, const lcs_hsmac_params &prm,
     run.ck.len3 = (double)(g.nx + 1) * (double)(g.ny + 1) * (double)(g.nz + 1);
     run.ck.dxmin = std::min(std::min(dx, dy), dz);
     run.ck.epsp = prm.epsp;
+    run.ck.noise = dv_noise<T>(g);
 
     const int last = 3 * ((prm.itrmax + 2) / 3) - 1;  // index of the last sweep the call can run
     auto may_end = [&](int n) { return n >= prm.itrmin ? 1 : 0; };
@@ -752,14 +769,18 @@ __global__ void __launch_bounds__(kDvBLx *kDvBNb)
     a.sum[1] = sum1;
     a.zc = B.dv_zc[NS - 1];
     a.px = dv_pitch(B.g, (int)sizeof(T));
-    double acc[NS];
-    Tile::run(a, it.bx, it.by, it.bz, lds, acc);
+    double acc[NS], nse;
+    Tile::run(a, it.bx, it.by, it.bz, lds, acc, nse);
     const int blk = (it.bz * B.dv_gy[NS - 1] + it.by) * B.dv_gx + it.bx;
     for (int s = 0; s < NS; s++)
         if (a.sum[s]) {
             const double v = block_sum(acc[s], red_lds);
             if (threadIdx.x == 0) B.part[(long)s * kMaxPartBlocks + blk] = v;
         }
+    if (MODE == kDvConstruct) {
+        const double v = block_sum(nse, red_lds);
+        if (threadIdx.x == 0) B.part[kDvNoiseSlot + blk] = v;
+    }
 }
 
 template <typename T>
@@ -811,18 +832,20 @@ __global__ void k_b_dv_check(const BoxRec *tab, const int *boxes, int slots, int
     const BoxRec &B = tab[boxes[blockIdx.x]];
     if (b_halted(B)) return;
     DevScalars *S = B.S;
+    double nse = (int)threadIdx.x < B.dv_tiles[0] ? B.part[kDvNoiseSlot + threadIdx.x] : 0.0;
     if (S->hs_done) return;
     const int cnt[5] = {B.dv_tiles[0], B.dv_tiles[1], B.dv_faces[0], B.dv_faces[1], B.dv_faces[2]};
     double acc = 0.0;
     for (int q = 0; q < 5; q++)
         if (slots >> q & 1)
             for (int m = threadIdx.x; m < cnt[q]; m += blockDim.x) acc += B.part[(long)q * kMaxPartBlocks + m];
-    const double s = block_sum(acc, lds);
+    for (int m = threadIdx.x + blockDim.x; m < B.dv_tiles[0]; m += blockDim.x) nse += B.part[kDvNoiseSlot + m];
+    const Geom &g = B.g;
+    const double len3 = (double)(g.nx + 1) * (double)(g.ny + 1) * (double)(g.nz + 1);
+    const double s = block_sum(acc / len3 + B.dv_noise * nse, lds);
     if (threadIdx.x == 0) {
-        const Geom &g = B.g;
-        const double len3 = (double)(g.nx + 1) * (double)(g.ny + 1) * (double)(g.nz + 1);
         const double dxmin = fmin(fmin(B.dx, B.dy), B.dz);
-        const double div = sqrt(s / len3);
+        const double div = sqrt(s);
         const int itr = itr_abs >= 0 ? itr_abs : S->hs_itr;
         S->hs_div = div;
         if (div * dxmin < epsp && itrmin <= itr) {
@@ -898,6 +921,7 @@ static int dv_record_t(Box &b, const lcs_hsmac_params &prm, int i, BoxRec &r, Dv
     const DvCoef<T> c = dv_coef<T>(g, prm.omega);
     const T v[9] = {c.k, c.cx, c.cy, c.cz, c.c0, c.c0l, c.dxi, c.dyi, c.dzi};
     for (int q = 0; q < 9; q++) r.dv_c[q] = (double)v[q];
+    r.dv_noise = dv_noise<T>(g);
     const int nplanes = g.nz + 2 * g.h;
     r.dv_gx = T1::tiles_x(g);
     r.dv_gy[0] = T1::tiles_y(g);

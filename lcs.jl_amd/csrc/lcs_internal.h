@@ -314,7 +314,7 @@ struct BoxRec {
     int dv;
     void *dv_mem;
     long dv_set;
-    double dv_c[9];
+    double dv_c[9], dv_noise;
     int dv_gx, dv_gy[2], dv_zc[2], dv_tiles[2], dv_faces[3];
     int dv_gxy, dv_fzc, dv_fin;
     DevProfile prof[kMaxProfiles];
