@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "lcs_internal.h"
+#include "lcs_hsmac_plan.h"
 #include "lcs_hsmac_xface.h"
 
 namespace lcs {
@@ -50,17 +51,24 @@ struct Server {
     }
 };
 
-// Device bytes a request will hold: 11 halo arrays (Us, Us2, P and the four
-// HSMAC partners), the compact buffer of the x-slab HSMAC pair, the reduction
-// partials, and per particle 17 properties plus staging, map and sort buffers.
-static size_t footprint(const lcs_request &r)
+constexpr int kServeGridRatio = 4;  // cells a particle cell of a run's profile
+
+// Device bytes a request will hold: seven halo arrays (Us, Us2, P); HSMAC's
+// (D, F) sets and planes in divergence form, or its four ping-pong partners and
+// the compact buffer of the x-slab pair; the reduction partials; per particle 17
+// properties plus staging, map and sort buffers, and the cell index.
+static size_t footprint(const lcs_request &r, const lcs_hsmac_params &hs)
 {
     const size_t es = r.dtype == LCS_F64 ? 8 : 4;
-    const size_t m = (size_t)(r.n + 6);
-    size_t bytes = 11 * m * m * m * es + sizeof(double) * (size_t)kPartSlots + (1u << 20);
-    bytes += (size_t)kXfVals * 2 * (size_t)(r.n - 1) * (size_t)(r.n - 1) * es;
-    const size_t np = (size_t)std::max<int64_t>(r.particles, 0);
+    const Geom g = make_geom(r.n, r.n, r.n, 3);
+    size_t bytes = 7 * (size_t)g.len * es + sizeof(double) * (size_t)kPartSlots + (1u << 20);
+    if (hsmac_takes_div(g, (int)es, hs))
+        bytes += dv_bytes(g, (int)es);
+    else
+        bytes += 4 * (size_t)g.len * es + (size_t)kXfVals * 2 * (size_t)(r.n - 1) * (size_t)(r.n - 1) * es;
+    const size_t np = (size_t)std::max<int64_t>(r.particles, 0), nc = (size_t)(r.n / kServeGridRatio + 2);
     bytes += np * (16 * es + 8 + 8 + es + 8 + 4 + 16 + 8);
+    if (np > 0) bytes += 2 * 8 * nc * nc * nc;
     return bytes;
 }
 
@@ -91,7 +99,7 @@ static int materialise(Server &S, Run &run)
     const int uvwp = (1 << LCS_FIELD_U) | (1 << LCS_FIELD_V) | (1 << LCS_FIELD_W) | (1 << LCS_FIELD_P);
     if ((rc = lcs_fill_ghost(run.box, uvwp, 3, 1))) return rc;
     if (r.particles > 0) {
-        lcs_particle_desc pd = {r.particles, r.particles, 0.0, 843.0, LCS_DRAG_LINEAR, 4};
+        lcs_particle_desc pd = {r.particles, r.particles, 0.0, 843.0, LCS_DRAG_LINEAR, kServeGridRatio};
         int prof = 0;
         if ((rc = lcs_particles_add(run.box, &pd, &prof))) return rc;
         if ((rc = lcs_init_particles(run.box, prof, r.seed ^ 0x9E3779B97F4A7C15ull, r.st_min, r.st_max, 0.5, 1)))
@@ -129,7 +137,7 @@ static int admit(Server &S)
 {
     for (auto it = S.queue.begin(); it != S.queue.end() && (int)S.live.size() < S.cfg.max_live;) {
         Run &run = S.runs[*it];
-        const size_t need = footprint(run.req);
+        const size_t need = footprint(run.req, S.cfg.hsmac);
         if (S.mem_used + need > S.cfg.memory_budget) {
             if (run.bypassed >= S.cfg.max_live) break;
             ++it;
@@ -207,8 +215,8 @@ int lcs_server_submit(lcs_server *server, const lcs_request *req, int64_t *id)
     int rc = check_request(*req);
     if (rc) return rc;
     Server &S = *SV(server);
-    if (footprint(*req) > S.cfg.memory_budget)
-        return fail(LCS_ERR_CAPACITY, "request needs " + std::to_string(footprint(*req)) +
+    if (footprint(*req, S.cfg.hsmac) > S.cfg.memory_budget)
+        return fail(LCS_ERR_CAPACITY, "request needs " + std::to_string(footprint(*req, S.cfg.hsmac)) +
                                           " bytes of device memory, more than the server's budget of " +
                                           std::to_string(S.cfg.memory_budget));
     Run run;
@@ -240,7 +248,7 @@ int lcs_server_step(lcs_server *server, int *n_live, int *n_finished)
                 if ((rc = lcs_batch_remove(S.batch, run.box))) return rc;
                 run.status = LCS_RUN_DONE;
                 run.finish_s = t;
-                S.mem_used -= std::min(S.mem_used, std::max(footprint(run.req), run.bytes));
+                S.mem_used -= std::min(S.mem_used, std::max(footprint(run.req, S.cfg.hsmac), run.bytes));
                 finished++;
             } else {
                 still.push_back(id);

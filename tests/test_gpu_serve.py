@@ -137,3 +137,19 @@ def test_invalid_requests_are_rejected():
     with pytest.raises(L.LCSArgumentError):
         S.submit(n=36, steps=3, seed=1, forcing="rc-energy")  # coarse size 8 must divide n
     S.close()
+
+
+@pytest.mark.parametrize("n,overlap", [(64, True), (64, False), (250, True), (256, True), (256, False)])
+def test_accounted_memory_covers_what_a_run_holds(n, overlap):
+    """The bytes admission counts for a run are at least those its box holds
+    once it has stepped: with the padded (D, F) sets and planes of HSMAC in
+    divergence form (rows are padded from n = 250 on), and with the ping-pong
+    partners and x-slab buffer of the in-place form."""
+    import lcs_mi355x as L
+    S = L.Server(max_live=1, hsmac=L.HSMAC(True, overlap, "red-black-fast", 1.7, 1e-3, 2, 6))
+    rid = S.submit(n, steps=3, seed=1, particles=1000)
+    S.step()
+    held, used = S.box(rid).nbytes(), S.counts()["memory_used"]
+    print(n, overlap, "held", held, "counted", used, flush=True)
+    assert held <= used <= 1.1 * held
+    S.close()
