@@ -503,7 +503,7 @@ struct DvRun {
         nz = (nplanes + a.zc - 1) / a.zc;
         const int blocks = (int)(cols * nz);
         const double cells = (double)g.cells() * sizeof(T);
-        ProfScope ps(b, MODE == kDvConstruct ? "hsmac_construct" : (NS == 2 ? "hsmac_sweep2" : "hsmac_sweep"),
+        ProfScope ps(b, MODE == kDvConstruct ? "hsmac_construct" : (NS == 2 ? "hsmac_div_sweep2" : "hsmac_div_sweep"),
                      (MODE == kDvConstruct ? 5.0 : 4.0) * cells);
         hipLaunchKernelGGL((k_dv_sweep<T, NS, MODE, LX, RW, NB, PF>), dim3(blocks), dim3(Tile::NT), 0, b.stream, a, gx,
                            gy, force ? 1 : 0, dt, b.S, b.part);
@@ -587,6 +587,7 @@ struct DvRun {
         LCS_HIP(hipGetLastError());
         return LCS_OK;
     }
+    double finish_bytes() const { return 9.0 * sizeof(T) * (double)b.g.cells(); }
     int finish(int when, int slot)
     {
         const Geom &g = b.g;
@@ -594,7 +595,7 @@ struct DvRun {
         dv_finish_grid(g, b.cus, gxy, zc, blocks);
         double *part = b.part + kPowerSlot;
         {
-            ProfScope ps(b, "hsmac_finish", 9.0 * sizeof(T) * g.cells());
+            ProfScope ps(b, "hsmac_finish", finish_bytes());
             if (force)
                 hipLaunchKernelGGL((k_dv_finish<T, true>), dim3(blocks), dim3(256), 0, b.stream, g, U, V, W, P, sets,
                                    (const T *)planes, c, dt, b.S, when, par, slot, nrefresh > 0 ? 1 : 0, zc, gxy, part);
@@ -684,6 +685,7 @@ static int hsmac_div_t(Box &b, void **Us, DtRef dt, const lcs_hsmac_params &prm,
                 // follows at once if so, and the host looks before it goes on
                 if ((rc = run.finish(1, slot)) || (rc = run.poll(done))) return rc;
                 if (done) return LCS_OK;
+                prof_uncount(b, "hsmac_finish", 1, run.finish_bytes());  // it found the call not done
             }
         }
         // d2 and d3: one pass unless the d2 sweep may end the iteration
@@ -700,7 +702,7 @@ static int hsmac_div_t(Box &b, void **Us, DtRef dt, const lcs_hsmac_params &prm,
             if ((rc = run.poll(done))) return rc;
             // the d3 sweep after a d2 sweep that ended the call did nothing
             if (done && may_end(n + 1) && b.S_host->hs_itr == n + 1)
-                prof_uncount(b, "hsmac_sweep", 1, 4.0 * sizeof(T) * (double)g.cells());
+                prof_uncount(b, "hsmac_div_sweep", 1, 4.0 * sizeof(T) * (double)g.cells());
         }
     }
     return run.finish(0, slot);
