@@ -314,7 +314,6 @@ __global__ void __launch_bounds__(TX *TY) k_rhs_flux(RhsArgs<T> a, DtRef dt)
 // planes a chunk: enough workgroups to cover the chip several times over, in
 // chunks of at least 8 planes (a chunk marches three planes more than it
 // writes), shorter where the box has too few cells for a workgroup on each CU
-template <typename T>
 static int rhs_chunk(const Geom &g, long cols)
 {
     const long least = std::max(2L, std::min(8L, cols * g.nz / 256));
@@ -331,7 +330,7 @@ static int rhs_tile_launch(Box &b, const RhsArgs<T> &a0, DtRef dt)
     if (g.h < 3) return fail(LCS_ERR_INVALID, "the fourth-order RHS needs halo_size >= 3");
     RhsArgs<T> a = a0;
     const int gx = (g.nx + TX - 1) / TX, gy = (g.ny + TY - 1) / TY;
-    a.zc = rhs_chunk<T>(g, (long)gx * gy);
+    a.zc = rhs_chunk(g, (long)gx * gy);
     const dim3 grid(gx, gy, (g.nz + a.zc - 1) / a.zc);
     const size_t lds = Tile::LDS_ELEMS * sizeof(T);
     if constexpr (FUSED) {

@@ -216,14 +216,16 @@ __device__ inline DvPair<T> dv_load2(const T *p)
 // planes at each end of a chunk.
 // A tile owns the OWN cells in the middle of its window of W: a multiple of a
 // 64-byte line, so stored row segments start and end on lines.
-template <typename T, int NS, int MODE, int LX, int RW, int NB, int PF = 2>
+template <typename T, int NS, int MODE, int LX, int RW, int NB>
 struct DvTile {
     using Win = DvWindow<(int)sizeof(T), NS, LX, RW, NB>;
     static constexpr int W = Win::W, OWN = Win::OWN, HX = Win::HX;
     static constexpr int ROWS = Win::ROWS, HY = Win::HY, HZ = 2 * NS, NT = NB * LX;
     static constexpr int EX = 2 * NS * 2 * NB * 2 * LX;  // exchange elements in LDS
     static_assert(RW % 2 == 0, "a block's first row keeps the parity of the tile's");
-    static_assert(PF % 2 == 0, "a register set serves steps of one parity");
+    // planes loaded ahead, one register set for steps of each parity (4 and 6
+    // sets: no faster at 32^3, 256^3 or 1000^3)
+    static constexpr int PF = 2;
     static_assert(HX >= 2 * NS && HX % 2 == 0, "halo of the window");
 
     __host__ __device__ static int tiles_x(const Geom &g) { return Win::tiles_x(g); }
@@ -360,7 +362,8 @@ struct DvTile {
         }
     }
 
-    // F of plane z (owned cells only are used)
+    // F of plane z: of every row of the window, though only the owned cells' is
+    // used (24 of 32 rows in a two-sweep pass)
     template <bool EXY>
     __device__ static inline void load_f(const DvArgs<T> &a, Th &th, int z, int e)
     {
@@ -385,7 +388,7 @@ struct DvTile {
             *p = v.v[0];
     }
 
-    // one plane; SET = step modulo PF, E = its parity: the red slot of row r on plane q is (E + r) & 1
+    // one plane; SET = E = the step's parity: the red slot of row r on plane q is (E + r) & 1
     template <int SET, bool EXY>
     __device__ static inline void step(const DvArgs<T> &a, T *lds, Th &th, int q)
     {
@@ -572,20 +575,6 @@ struct DvTile {
             __syncthreads();
             step<1, EXY>(a, lds, th, q + 1);
             __syncthreads();
-            if constexpr (PF >= 4) {
-                if (q + 2 > q1) break;
-                step<PF >= 4 ? 2 : 0, EXY>(a, lds, th, q + 2);
-                __syncthreads();
-                step<PF >= 4 ? 3 : 1, EXY>(a, lds, th, q + 3);
-                __syncthreads();
-            }
-            if constexpr (PF >= 6) {
-                if (q + 4 > q1) break;
-                step<PF >= 6 ? 4 : 0, EXY>(a, lds, th, q + 4);
-                __syncthreads();
-                step<PF >= 6 ? 5 : 1, EXY>(a, lds, th, q + 5);
-                __syncthreads();
-            }
         }
     }
 

@@ -23,11 +23,11 @@ struct DvSets {
 
 // (The FP32 construct pass of 512 threads needs 129 registers left alone; at
 // 128 two workgroups share a CU, as before it summed the rounding terms.)
-template <typename T, int NS, int MODE, int LX, int RW, int NB, int PF>
+template <typename T, int NS, int MODE, int LX, int RW, int NB>
 __global__ void __launch_bounds__(LX *NB, MODE == kDvConstruct && sizeof(T) == 4 ? 4 : 1)
     k_dv_sweep(DvArgs<T> a, int gx, int gy, int force, DtRef dt, DevScalars *S, double *part)
 {
-    using Tile = DvTile<T, NS, MODE, LX, RW, NB, PF>;
+    using Tile = DvTile<T, NS, MODE, LX, RW, NB>;
     __shared__ __align__(16) T lds[Tile::EX];
     __shared__ double red_lds[16];
     if (MODE != kDvConstruct && S->hs_done) return;
@@ -472,10 +472,10 @@ struct DvRun {
     bool force = false;
     DvCheck ck;
 
-    template <int NS, int MODE, int LX, int RW, int NB, int PF = 2>
+    template <int NS, int MODE, int LX, int RW, int NB>
     int sweep(int k0, int k1, int sum0, int sum1)
     {
-        using Tile = DvTile<T, NS, MODE, LX, RW, NB, PF>;
+        using Tile = DvTile<T, NS, MODE, LX, RW, NB>;
         const Geom &g = b.g;
         DvArgs<T> a;
         a.g = g;
@@ -495,7 +495,7 @@ struct DvRun {
         a.sum[1] = sum1;
         const int gx = Tile::tiles_x(g), gy = Tile::tiles_y(g), nplanes = g.nz + 2 * g.h;
         const long cols = (long)gx * gy;
-        const void *k = (const void *)k_dv_sweep<T, NS, MODE, LX, RW, NB, PF>;
+        const void *k = (const void *)k_dv_sweep<T, NS, MODE, LX, RW, NB>;
         int per_cu = 1, rc = kernel_setup(k, Tile::NT, 0, &per_cu);
         if (rc) return rc;
         int nz = dv_chunks(cols, nplanes, 4 * NS, (long)b.cus * per_cu);
@@ -505,7 +505,7 @@ struct DvRun {
         const double cells = (double)g.cells() * sizeof(T);
         ProfScope ps(b, MODE == kDvConstruct ? "hsmac_construct" : (NS == 2 ? "hsmac_div_sweep2" : "hsmac_div_sweep"),
                      (MODE == kDvConstruct ? 5.0 : 4.0) * cells);
-        hipLaunchKernelGGL((k_dv_sweep<T, NS, MODE, LX, RW, NB, PF>), dim3(blocks), dim3(Tile::NT), 0, b.stream, a, gx,
+        hipLaunchKernelGGL((k_dv_sweep<T, NS, MODE, LX, RW, NB>), dim3(blocks), dim3(Tile::NT), 0, b.stream, a, gx,
                            gy, force ? 1 : 0, dt, b.S, b.part);
         LCS_HIP(hipGetLastError());
         if (MODE == kDvConstruct) ck.nnoise = blocks;
@@ -528,12 +528,15 @@ struct DvRun {
         // the rows a workgroup can hold.
         const long sy = b.g.sy;
         if constexpr (sizeof(T) == 8) {
-            if (NS == 1 && MODE == kDvPlain && sy >= 256) return sweep<NS, MODE, 32, 2, 24>(k0, k1, sum0, sum1);
+            if constexpr (NS == 1 && MODE == kDvPlain)
+                if (sy >= 256) return sweep<NS, MODE, 32, 2, 24>(k0, k1, sum0, sum1);
             return sweep<NS, MODE, 32, 2, 16>(k0, k1, sum0, sum1);
         } else {
             if (sy < 200) return sweep<NS, MODE, 32, 2, 16>(k0, k1, sum0, sum1);
-            if (NS == 2 && sy < 512) return sweep<NS, MODE, 64, 2, 12>(k0, k1, sum0, sum1);
-            if (NS == 1 && MODE == kDvPlain && sy >= 512) return sweep<NS, MODE, 64, 4, 12>(k0, k1, sum0, sum1);
+            if constexpr (NS == 2)
+                if (sy < 512) return sweep<NS, MODE, 64, 2, 12>(k0, k1, sum0, sum1);
+            if constexpr (NS == 1 && MODE == kDvPlain)
+                if (sy >= 512) return sweep<NS, MODE, 64, 4, 12>(k0, k1, sum0, sum1);
             return sweep<NS, MODE, 64, 2, 16>(k0, k1, sum0, sum1);
         }
     }
@@ -628,15 +631,6 @@ int dv_buffers(Box &b)
     b.bytes += bytes;
     return LCS_OK;
 }
-
-// Groups carried on D and F before they go into the velocity and D is formed
-// anew.  Most calls end in the third group; in calls of hundreds of sweeps
-// (the first steps from a synthetic field) the rounding of D and of F, which
-// accumulates over the sweeps, would exceed that of the velocity's own updates:
-// after eight 256^3 FP32 steps with 300-sweep calls the fields were 1.4e-6 off
-// FP64 without the limit, 0.6e-6 with it and 1.0e-6 with every sweep on the
-// velocity (the velocity alone 0.12e-6 with it, 0.5e-6 with every sweep on it).
-// (kDvGroups)
 
 template <typename T>
 static int hsmac_div_t(Box &b, void **Us, DtRef dt, const lcs_hsmac_params &prm, int slot, bool lf_deferred)
