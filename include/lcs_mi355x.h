@@ -409,8 +409,8 @@ int lcs_batch_set_graphs(lcs_batch *batch, int on);
  * segmented = eager or segment launches.  Any pointer may be NULL. */
 int lcs_batch_graph_stats(lcs_batch *batch, int64_t *whole, int64_t *gated, int64_t *segmented);
 /* No counterpart in the reference (its kernels launch one workgroup per
- * block).  cus < 0: each batched HSMAC sweep runs as a persistent grid, as
- * many workgroups as the device holds at once, each walking the tile table
+ * block).  cus < 0: each batched HSMAC sweep on the velocity (not those of boxes
+ * in divergence form, see lcs_batch_set_tiles) runs as a persistent grid, as many workgroups as the device holds at once, each walking the tile table
  * (tiles b, b + G, b + 2G, ...); cus > 0: the grid that many CUs hold (at most
  * the device's); cus = 0 (default): one workgroup per tile.  Results are the
  * same in every case (a tile's arithmetic does not depend on the workgroup
