@@ -42,7 +42,6 @@
 // FP32, U in [0, 1): floor 3.2e-8 / dx, the returned velocity's 2.5e-8 to 3e-8).
 #pragma once
 
-#include "lcs_device.h"
 #include "lcs_hsmac_plan.h"
 #include "lcs_hsmac_tile.h"
 #include "lcs_internal.h"
@@ -88,7 +87,7 @@ inline double dv_noise(const Geom &g)
 }
 // a batch record's coefficients (the T values, stored as doubles)
 template <typename T>
-__device__ inline DvCoef<T> dv_coef_rec(const BoxRec &B)
+__host__ __device__ inline DvCoef<T> dv_coef_rec(const BoxRec &B)
 {
     DvCoef<T> c;
     c.k = T(B.dv_c[0]);
@@ -104,9 +103,9 @@ __device__ inline DvCoef<T> dv_coef_rec(const BoxRec &B)
 }
 // D of a cell after its own correction
 template <typename T>
-__device__ inline T dv_self(const DvCoef<T> &c, T d, T dp)
+__host__ __device__ inline T dv_self(const DvCoef<T> &c, T d, T dp)
 {
-    return __builtin_elementwise_fma(c.c0, dp, __builtin_elementwise_fma(c.c0l, dp, d));
+    return std::fma(c.c0, dp, std::fma(c.c0l, dp, d));
 }
 
 enum { kDvPlain = 0, kDvConstruct = 1 };
@@ -129,7 +128,7 @@ struct DvArgs {
 // plane (array indices x, y, z): Do, Fo the set the core sweep read, Dn, Fn the
 // one it wrote.  accumulate: seams of an earlier refresh of the call are kept.
 template <typename T>
-__device__ inline void dv_refresh_cell(const Geom &g, const DvCoef<T> &c, const DvPlanes &pl, const T *Do, const T *F,
+__host__ __device__ inline void dv_refresh_cell(const Geom &g, const DvCoef<T> &c, const DvPlanes &pl, const T *Do, const T *F,
                                        T *Dn, T *Fn, T *P, T *pn, T dti, int accumulate, int x, int y, int z)
 {
     const int h = g.h, nx = g.nx, ny = g.ny, nz = g.nz;
@@ -173,6 +172,7 @@ __device__ inline void dv_refresh_cell(const Geom &g, const DvCoef<T> &c, const 
 }
 
 // neighbouring lane's value across the wave; lanes past its ends read 0
+#ifdef __HIPCC__
 template <int UP>
 __device__ inline float dv_lane(float v)
 {
@@ -185,6 +185,13 @@ __device__ inline double dv_lane(double v)
     const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), UP ? 0x130 : 0x138, 0xf, 0xf, true);
     return __hiloint2double(hi, lo);
 }
+#endif
+// member m of the neighbouring lane's state as it was before this step
+#ifdef __HIP_DEVICE_COMPILE__
+#define DV_LANE(UP, m) dv_lane<UP>(th.m)
+#else
+#define DV_LANE(UP, m) (th.lane[UP] ? th.lane[UP]->m : T(0))
+#endif
 
 template <typename T>
 struct DvPair {
@@ -192,7 +199,7 @@ struct DvPair {
 };
 // two neighbouring elements of a row (rows start at any element)
 template <typename T>
-__device__ inline DvPair<T> dv_load2(const T *p)
+__host__ __device__ inline DvPair<T> dv_load2(const T *p)
 {
     DvPair<T> r;
     __builtin_memcpy(&r, p, sizeof(r));
@@ -232,6 +239,9 @@ struct DvTile {
     __host__ __device__ static int tiles_y(const Geom &g) { return Win::tiles_y(g); }
 
     struct Th {
+#ifndef __HIP_DEVICE_COMPILE__
+        const Th *lane[2];      // host harness: states of the lanes below and above before the step
+#endif
         int X, xo, b, lx;       // first cell of the lane, clamped load offset, block, lane
         int Y;                  // first row of the block
         int wx0, wy0, ox0, ox1, oy0, oy1, zo0, zo1;
@@ -254,15 +264,16 @@ struct DvTile {
         T nse;  // construct: sum of dxi^2 U^2 + dyi^2 V^2 + dzi^2 W^2 (a lane that owns one of its rows counts both)
     };
 
-    __device__ static inline int clampi(int v, int hi) { return v < 0 ? 0 : (v > hi ? hi : v); }
+    __host__ __device__ static inline int mini(int a, int b) { return a < b ? a : b; }
+    __host__ __device__ static inline int clampi(int v, int hi) { return v < 0 ? 0 : (v > hi ? hi : v); }
 
     // returns whether any cell of the window lies outside the core (2:n) in x or y
-    __device__ static bool init(const DvArgs<T> &a, int bx, int by, int bz, Th &th)
+    __host__ __device__ static bool init(const DvArgs<T> &a, int bx, int by, int bz, int tid, Th &th)
     {
         const Geom &g = a.g;
         const int gx = tiles_x(g), gy = tiles_y(g);
-        th.b = (int)threadIdx.x / LX;
-        th.lx = (int)threadIdx.x % LX;
+        th.b = tid / LX;
+        th.lx = tid % LX;
         th.ox0 = bx * OWN;
         th.ox1 = bx == gx - 1 ? (int)g.sx : th.ox0 + OWN;
         th.wx0 = bx == 0 ? 0 : th.ox0 - HX;
@@ -270,10 +281,10 @@ struct DvTile {
         th.oy0 = by == 0 ? 0 : th.wy0 + HY;
         th.oy1 = by == gy - 1 ? (int)g.sy : th.wy0 + ROWS - HY;
         th.zo0 = bz * a.zc;
-        th.zo1 = min(g.nz + 2 * g.h, th.zo0 + a.zc);
+        th.zo1 = mini(g.nz + 2 * g.h, th.zo0 + a.zc);
         th.X = th.wx0 + 2 * th.lx;
         th.Y = th.wy0 + th.b * RW;
-        th.xo = min(th.X, (int)g.sx - 2);
+        th.xo = mini(th.X, (int)g.sx - 2);
         th.own = 0;
         th.cnt = 0;
         const int h = g.h;
@@ -316,20 +327,20 @@ struct DvTile {
 
     // element offset of row r's load in its plane of row pitch px
     template <bool EXY>
-    __device__ static inline int row_off(const Geom &g, const Th &th, int r, int px)
+    __host__ __device__ static inline int row_off(const Geom &g, const Th &th, int r, int px)
     {
-        const int y = EXY ? min(th.Y + r, (int)g.sy - 1) : th.Y + r;
+        const int y = EXY ? mini(th.Y + r, (int)g.sy - 1) : th.Y + r;
         return y * px + th.xo;
     }
     // a lane whose first cell is the row's last element loaded one element early
     template <bool EXY>
-    __device__ static inline void fix_end(const Geom &g, const Th &th, DvPair<T> &p)
+    __host__ __device__ static inline void fix_end(const Geom &g, const Th &th, DvPair<T> &p)
     {
         if (EXY && th.X == (int)g.sx - 1) p.v[0] = p.v[1];
     }
 
     template <bool EXY>
-    __device__ static inline void load_d(const DvArgs<T> &a, Th &th, int q, int e)
+    __host__ __device__ static inline void load_d(const DvArgs<T> &a, Th &th, int q, int e)
     {
         const Geom &g = a.g;
         const int sz = g.nz + 2 * g.h;
@@ -337,7 +348,7 @@ struct DvTile {
         if constexpr (MODE == kDvConstruct) {
             const long base = (long)z * (g.sx * g.sy);
             const T *U = a.U + base, *V = a.V + base, *Wz = a.W + base;
-            const int xm = max(min(th.X, (int)g.sx) - 1, 0);
+            const int xm = clampi(th.X - 1, (int)g.sx - 1);
 #pragma unroll
             for (int r = 0; r < RW; r++) {
                 const int o = row_off<EXY>(g, th, r, (int)g.sx);
@@ -349,7 +360,7 @@ struct DvTile {
                 th.w[e][r] = dv_load2(Wz + o);
                 fix_end<EXY>(g, th, th.w[e][r]);
             }
-            const int ym = min(max(th.Y - 1, 0), (int)g.sy - 1);
+            const int ym = clampi(th.Y - 1, (int)g.sy - 1);
             th.v[e][0] = dv_load2(V + ym * (int)g.sx + th.xo);
             fix_end<EXY>(g, th, th.v[e][0]);
         } else {
@@ -365,7 +376,7 @@ struct DvTile {
     // F of plane z: of every row of the window, though only the owned cells' is
     // used (24 of 32 rows in a two-sweep pass)
     template <bool EXY>
-    __device__ static inline void load_f(const DvArgs<T> &a, Th &th, int z, int e)
+    __host__ __device__ static inline void load_f(const DvArgs<T> &a, Th &th, int z, int e)
     {
         if constexpr (MODE == kDvConstruct) return;
         const Geom &g = a.g;
@@ -379,7 +390,7 @@ struct DvTile {
     }
 
     // store a pair of owned cells
-    __device__ static inline void store2(T *p, const Th &th, int r, const DvPair<T> &v)
+    __host__ __device__ static inline void store2(T *p, const Th &th, int r, const DvPair<T> &v)
     {
         const unsigned m = th.own >> (2 * r) & 3u;
         if (m == 3u)
@@ -390,7 +401,7 @@ struct DvTile {
 
     // one plane; SET = E = the step's parity: the red slot of row r on plane q is (E + r) & 1
     template <int SET, bool EXY>
-    __device__ static inline void step(const DvArgs<T> &a, T *lds, Th &th, int q)
+    __host__ __device__ static inline void step(const DvArgs<T> &a, T *lds, Th &th, int q)
     {
         constexpr int E = SET & 1;
         const Geom &g = a.g;
@@ -442,7 +453,7 @@ struct DvTile {
             // rows of the neighbouring blocks (dp of the last step)
             const T *ein = xin + s * (4 * NB * LX);
             T *eout = xout + s * (4 * NB * LX);
-            const int bm = max(th.b - 1, 0), bpl = min(th.b + 1, NB - 1);
+            const int bm = clampi(th.b - 1, NB - 1), bpl = clampi(th.b + 1, NB - 1);
             const T rdn = ein[(bm * 2 + 1) * LX + th.lx], rup = ein[bpl * 2 * LX + th.lx];
             const T bdn = ein[2 * NB * LX + (bm * 2 + 1) * LX + th.lx];
             const T bup = ein[2 * NB * LX + bpl * 2 * LX + th.lx];
@@ -459,7 +470,7 @@ struct DvTile {
             for (int r = 0; r < RW; r++) {
                 const int sr = (E + r + 1) & 1;  // red slot on plane zr-1
                 const T own = th.rp[s][r];
-                const T oth = sr == 0 ? dv_lane<1>(own) : dv_lane<0>(own);
+                const T oth = sr == 0 ? DV_LANE(1, rp[s][r]) : DV_LANE(0, rp[s][r]);
                 const T dn = r > 0 ? th.rp[s][r > 0 ? r - 1 : 0] : rdn;
                 const T up = r < RW - 1 ? th.rp[s][r < RW - 1 ? r + 1 : r] : rup;
                 T B = s == 0 ? th.bq0[r] : th.bq1[1][r];
@@ -474,7 +485,7 @@ struct DvTile {
             for (int r = 0; r < RW; r++) {
                 const int sr = (E + r) & 1;  // red slot on plane zr-2
                 const T own = th.bp[s][r];
-                const T oth = sr == 0 ? dv_lane<0>(own) : dv_lane<1>(own);
+                const T oth = sr == 0 ? DV_LANE(0, bp[s][r]) : DV_LANE(1, bp[s][r]);
                 const T dn = r > 0 ? th.bp[s][r > 0 ? r - 1 : 0] : bdn;
                 const T up = r < RW - 1 ? th.bp[s][r < RW - 1 ? r + 1 : r] : bup;
                 R[r] = ((th.rq[s][1][r] - c.cx * (own + oth)) - c.cy * (dn + up)) - c.cz * (th.bpp[s][r] + bn[s][r]);
@@ -549,15 +560,19 @@ struct DvTile {
         }
     }
 
+    // the first step's plane: red cells have even i+j+k, and it is chosen so that
+    // the red slot of row r on plane q is (step parity + r) & 1
+    __host__ __device__ static inline int first(const DvArgs<T> &a, const Th &th)
+    {
+        const int q = th.zo0 - HZ > 0 ? th.zo0 - HZ : 0;
+        return (th.wx0 + th.wy0 + q + a.g.h + 1) & 1 ? q - 1 : q;
+    }
+    __host__ __device__ static inline int last(const Th &th) { return th.zo1 - 1 + HZ; }
+    // loads ahead of step q
     template <bool EXY>
-    __device__ static inline void march(const DvArgs<T> &a, T *lds, Th &th)
+    __host__ __device__ static inline void prologue(const DvArgs<T> &a, Th &th, int q)
     {
         const Geom &g = a.g;
-        // red cells have even i+j+k; the first step is chosen so that the red
-        // slot of row r on plane q is (step parity + r) & 1
-        int q = max(0, th.zo0 - HZ);
-        if ((th.wx0 + th.wy0 + q + g.h + 1) & 1) q--;
-        const int q1 = th.zo1 - 1 + HZ;
 #pragma unroll
         for (int e = 0; e < PF; e++) load_d<EXY>(a, th, q + e, e);
         if constexpr (MODE == kDvConstruct) {  // W below the first plane
@@ -570,6 +585,14 @@ struct DvTile {
         }
 #pragma unroll
         for (int e = 0; e < PF; e++) load_f<EXY>(a, th, q - 2 * (NS - 1) - 1 + e, e);
+    }
+#ifdef __HIPCC__
+    template <bool EXY>
+    __device__ static inline void march(const DvArgs<T> &a, T *lds, Th &th)
+    {
+        int q = first(a, th);
+        const int q1 = last(th);
+        prologue<EXY>(a, th, q);
         for (; q <= q1; q += PF) {
             step<0, EXY>(a, lds, th, q);
             __syncthreads();
@@ -582,7 +605,7 @@ struct DvTile {
     __device__ static inline void run(const DvArgs<T> &a, int bx, int by, int bz, T *lds, double acc[NS], double &nse)
     {
         Th th;
-        const bool edge = init(a, bx, by, bz, th);
+        const bool edge = init(a, bx, by, bz, (int)threadIdx.x, th);
         for (int t = threadIdx.x; t < EX; t += NT) lds[t] = T(0);
         __syncthreads();
         if (edge)
@@ -592,6 +615,42 @@ struct DvTile {
 #pragma unroll
         for (int s = 0; s < NS; s++) acc[s] = th.acc[s];
         nse = th.own ? (double)th.nse : 0.0;
+    }
+#endif
+
+    // One workgroup for a host harness, step by step in the kernel's barrier order:
+    // th and was hold NT states each.
+    template <bool EXY>
+    static void emulate_march(const DvArgs<T> &a, T *lds, Th *th, Th *was)
+    {
+        const int q0 = first(a, th[0]), q1 = last(th[0]);
+        for (int t = 0; t < NT; t++) prologue<EXY>(a, th[t], q0);
+        for (int q = q0; q <= q1 + (q1 - q0 + 1) % PF; q++) {
+            for (int t = 0; t < NT; t++) was[t] = th[t];
+            for (int t = 0; t < NT; t++) {
+                th[t].lane[0] = t % 64 > 0 ? was + t - 1 : nullptr;
+                th[t].lane[1] = t % 64 < 63 && t + 1 < NT ? was + t + 1 : nullptr;
+                if ((q - q0) % PF == 0)
+                    step<0, EXY>(a, lds, th[t], q);
+                else
+                    step<1, EXY>(a, lds, th[t], q);
+            }
+        }
+    }
+    static void emulate_block(const DvArgs<T> &a, int bx, int by, int bz, T *lds, Th *th, Th *was, double acc[NS],
+                              double &nse)
+    {
+        bool edge = false;
+        for (int t = 0; t < NT; t++) edge = init(a, bx, by, bz, t, th[t]);
+        for (int t = 0; t < EX; t++) lds[t] = T(0);
+        if (edge)
+            emulate_march<true>(a, lds, th, was);
+        else
+            emulate_march<false>(a, lds, th, was);
+        for (int t = 0; t < NT; t++) {
+            for (int s = 0; s < NS; s++) acc[s] += th[t].acc[s];
+            if (th[t].own) nse += (double)th[t].nse;
+        }
     }
 };
 
