@@ -265,6 +265,7 @@ struct DvTile {
     };
 
     __host__ __device__ static inline int mini(int a, int b) { return a < b ? a : b; }
+    __host__ __device__ static inline int maxi(int a, int b) { return a > b ? a : b; }
     __host__ __device__ static inline int clampi(int v, int hi) { return v < 0 ? 0 : (v > hi ? hi : v); }
 
     // returns whether any cell of the window lies outside the core (2:n) in x or y
@@ -348,7 +349,7 @@ struct DvTile {
         if constexpr (MODE == kDvConstruct) {
             const long base = (long)z * (g.sx * g.sy);
             const T *U = a.U + base, *V = a.V + base, *Wz = a.W + base;
-            const int xm = clampi(th.X - 1, (int)g.sx - 1);
+            const int xm = maxi(mini(th.X, (int)g.sx) - 1, 0);
 #pragma unroll
             for (int r = 0; r < RW; r++) {
                 const int o = row_off<EXY>(g, th, r, (int)g.sx);
@@ -360,7 +361,7 @@ struct DvTile {
                 th.w[e][r] = dv_load2(Wz + o);
                 fix_end<EXY>(g, th, th.w[e][r]);
             }
-            const int ym = clampi(th.Y - 1, (int)g.sy - 1);
+            const int ym = mini(maxi(th.Y - 1, 0), (int)g.sy - 1);
             th.v[e][0] = dv_load2(V + ym * (int)g.sx + th.xo);
             fix_end<EXY>(g, th, th.v[e][0]);
         } else {
